@@ -88,20 +88,22 @@ __device__ __forceinline__ u32 encode_planes(W& w, const UInt* u, u32 maxbits, u
 }
 
 // decoding mirror (src/template/decode.c:78-278); u receives the
-// coefficients' bits, zero where no plane was coded
+// coefficients' bits, zero where no plane was coded.  Once no lane wants a
+// plane none wants a lower one, which ends the loop.
 template <int N, typename R>
 __device__ __forceinline__ void decode_half(PlaneDecoder<N>& pd, R& r, PlaneVec& lo, PlaneVec& hi,
                                             u32 base)
 {
+  lo = PlaneVec(0);
+  hi = PlaneVec(0);
   for (int k = 31; k >= 0; k--) {
     const bool act = pd.wants(base + (u32)k);
+    if (!wave_any(act))
+      break;
     u64 x = 0;
-    if (wave_any(act)) {
-      if (act)
-        x = pd.plane(r);
-    }
-    // every plane is written (zero when not coded); the plane number is
-    // uniform, which readfirstlane states to the compiler
+    if (act)
+      x = pd.plane(r);
+    // the plane number is uniform, which readfirstlane states to the compiler
     const int ku = __builtin_amdgcn_readfirstlane(k);
     lo[ku] = (u32)x;
     hi[ku] = (u32)(x >> 32);
