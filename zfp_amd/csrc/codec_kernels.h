@@ -36,6 +36,20 @@
 
 namespace zfphip {
 
+// LDS operations of the lanes of one wave, ordered before what follows
+ZH_INLINE void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+} // namespace zfphip
+
+#include "codec_quad4.h"
+
+namespace zfphip {
+
 // ENC_FIXED_PLAIN: fixed rate with every block range word-aligned, so each
 // lane owns whole words and stores them without atomics; ENC_FIXED_AT: the
 // same with block b placed at bit offset + boffs[b] (chosen slots)
@@ -98,14 +112,6 @@ k_encode(const S* __restrict__ data, Geom g, u32 nblocks, Params z,
   w.begin(out, start, end);
   encode_any<S, D, REV>(w, data, g, bc, z);
   w.finish();
-}
-
-// LDS operations of the lanes of one wave, ordered before what follows
-ZH_INLINE void wave_lds_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Word runs between the lanes' LDS slots (nw words each, slot stride
@@ -343,10 +349,9 @@ k_encode_waves(const S* __restrict__ data, Geom g, u32 nblocks, Params z, u64* _
 //   k_encode_blocks  codes block b into its own bw words of `stage` (from
 //                    bit 0, plain stores) and writes its length;
 //   exclusive scan   of the lengths: the block offsets;
-//   k_place_blocks   k_encode_waves with the staged bits in place of a
-//                    second coding: each wave assembles its blocks' bits in
-//                    LDS and stores whole words, OR-ing only its two edge
-//                    words (zeroed by k_prepare).
+//   k_clear_edges, k_place_blocks   the staged bits to their places.
+//
+// 4D lossy blocks are coded by k_encode_quad in place of k_encode_blocks.
 template <typename S, int D, bool REV>
 __global__ void __launch_bounds__(256)
 k_encode_blocks(const S* __restrict__ data, Geom g, u32 nblocks, Params z, u64* __restrict__ stage,
@@ -366,60 +371,52 @@ k_encode_blocks(const S* __restrict__ data, Geom g, u32 nblocks, Params z, u64* 
     lens[nblocks] = 0; // so that the exclusive scan's last entry is the total
 }
 
+// Each block's staged bits shifted to their place in the stream, 16 lanes per
+// block, so that a lane group loads and stores runs of 128 bytes; words that
+// two blocks share are OR-ed into memory k_clear_edges zeroed.  It moves the
+// stream's bytes twice: bound by HBM.
 template <int UNUSED = 0>
 __global__ void __launch_bounds__(256)
 k_place_blocks(const u64* __restrict__ stage, u32 bw, u32 nblocks, u64* __restrict__ out, u64 offset,
-               const u64* __restrict__ boffs, u32 wcap)
+               const u64* __restrict__ boffs)
 {
-  extern __shared__ u64 wstage[];
-  const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
-  const u32 lane = threadIdx.x & 63u;
-  const u32 t0 = t - lane;
-  if (t0 >= nblocks)
-    return; // the whole wave lies past the field
-  const u32 tl = umin(t0 + 63u, nblocks - 1u);
-  const u64 first = offset + boffs[t0], end = offset + boffs[tl + 1];
-  const u64 wlo = first >> 6, whi = (end + 63) >> 6;
-  const bool staged = whi - wlo <= wcap;
-  const u32 nw = staged ? (u32)(whi - wlo) : 0u;
-  u64* st = wstage + (u64)(threadIdx.x >> 6) * wcap;
-  for (u32 i = lane; i < nw; i += 64)
-    st[i] = 0;
-  wave_lds_sync();
-  if (t < nblocks) {
-    WaveWriter w;
-    w.out = out; w.st = st; w.wbase = wlo; w.staged = staged;
-    w.lo = offset + boffs[t]; w.hi = offset + boffs[t + 1];
-    w.wi = w.lo >> 6; w.fill = (u32)(w.lo & 63); w.acc = 0;
-    const u64 len = boffs[t + 1] - boffs[t];
-    const u64* src = stage + (u64)t * bw;
-    // eight loads in flight at a time (words of the block's own stride,
-    // always readable), then their bits in order
-    for (u64 i0 = 0; 64 * i0 < len; i0 += 8) {
-      u64 v[8];
-#pragma unroll
-      for (u32 j = 0; j < 8; j++)
-        v[j] = i0 + j < bw ? src[i0 + j] : 0ull;
-#pragma unroll
-      for (u32 j = 0; j < 8; j++) {
-        const u64 at = 64 * (i0 + j);
-        if (at < len) {
-          const u32 n = (u32)(len - at < 64 ? len - at : 64);
-          w.put(v[j] & lowmask(n), n);
-        }
-      }
-    }
-    w.finish();
-  }
-  wave_lds_sync();
-  for (u32 i = lane; i < nw; i += 64) {
-    const u64 v = st[i];
-    const bool edge = (i == 0 && (first & 63)) || (i + 1 == nw && (end & 63));
-    if (!edge)
-      out[wlo + i] = v;
+  const u32 t = (u32)(((u64)blockIdx.x * blockDim.x + threadIdx.x) >> 4);
+  if (t >= nblocks)
+    return;
+  const u64 first = boffs[t];
+  const u32 len = (u32)(boffs[t + 1] - first);
+  const u64 G = offset + first;
+  const u32 s = (u32)(G & 63), lw = (len + 63) >> 6, nout = (s + len + 63) >> 6;
+  const u64 tail = len & 63 ? lowmask(len & 63) : ~0ull; // bits of the last staged word
+  const u64* src = stage + (u64)t * bw;
+  u64* dst = out + (G >> 6);
+  for (u32 j = threadIdx.x & 15u; j < nout; j += 16) {
+    u64 cur = j < lw ? src[j] : 0ull, prev = j ? src[j - 1] : 0ull;
+    cur &= j + 1 == lw ? tail : ~0ull;
+    prev &= j == lw ? tail : ~0ull;
+    const u64 v = s ? (cur << s) | (prev >> (64 - s)) : cur;
+    const bool shared = (j == 0 && s) || (j + 1 == nout && ((s + len) & 63));
+    if (!shared)
+      dst[j] = v;
     else if (v)
-      atomicOr((unsigned long long*)(out + wlo + i), (unsigned long long)v);
+      atomicOr((unsigned long long*)(dst + j), (unsigned long long)v);
   }
+}
+
+// Zeroes the words in which a block starts or the stream ends off a word
+// boundary, keeping the bits below `offset`: those that k_place_blocks ORs
+// into.  (Blocks that start in one word store the same value there.)
+template <int UNUSED = 0>
+__global__ void __launch_bounds__(256)
+k_clear_edges(u64* __restrict__ out, u64 offset, const u64* __restrict__ boffs, u32 nblocks)
+{
+  const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t > nblocks)
+    return;
+  const u64 G = offset + boffs[t], w = G >> 6;
+  if (!(G & 63))
+    return;
+  out[w] = w == offset >> 6 ? out[w] & lowmask((u32)(offset & 63)) : 0ull;
 }
 
 // Bits one block can take in the stream's mode: the per-block term of
@@ -1013,7 +1010,8 @@ int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out
   // 32 words); not for the caller's workspace (no allocation, a fixed set of
   // passes)
   const u32 bw = (block_bits_bound<S, D, REV>(z) + 63) / 64;
-  if (stream_order && !ws && bw >= 1 && bw <= 32 && d.nblocks > 0) {
+  constexpr bool QUAD = D == 4 && !REV; // 4D lossy blocks go over four lanes
+  if constexpr (D < 4) if (stream_order && !ws && bw >= 1 && bw <= 32 && d.nblocks > 0) {
     u64 total = 0;
     rc = encode_once<S, D, REV>(d, data, z, out, offset, offs, bw, &total, st);
     if (rc == ZFP_HIP_OK) {
@@ -1030,20 +1028,40 @@ int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out
       return rc;
   }
   // longer blocks in stream order: each coded once into a staging stride
-  // of bw words when those fit in device memory (k_encode_blocks), else
-  // a length pass now and a second coding in the write pass
+  // of bw words when those fit in device memory (k_encode_quad for 4D lossy
+  // blocks, else k_encode_blocks), else a length pass now and a second
+  // coding in the write pass
   u64* bstage = nullptr;
-  if (stream_order && !ws && bw > 32 && d.nblocks > 0) {
+  if (stream_order && !ws && (bw > 32 || (D == 4 && bw >= 1)) && d.nblocks > 0) {
     void* tp;
     if (g_stage.get((u64)d.nblocks * bw * sizeof(u64), &tp) == ZFP_HIP_OK)
       bstage = (u64*)tp;
   }
-  if (bstage)
-    hipLaunchKernelGGL((k_encode_blocks<S, D, REV>), dim3(grid), dim3(BS), 0, st, (const S*)data, d.g, d.nblocks,
-                       z, bstage, lens, bw);
-  else
-    hipLaunchKernelGGL((k_encode<S, D, ENC_LENGTH, REV>), dim3(grid), dim3(BS), 0, st, (const S*)data, d.g,
-                       d.nblocks, z, out, offset, (const u64*)nullptr, lens);
+  if (bstage) {
+    if constexpr (QUAD)
+      hipLaunchKernelGGL((k_encode_quad<S>), dim3(grid_for(d.nblocks, 16)), dim3(64), 0, st, (const S*)data, d.g,
+                         d.nblocks, z, bstage, lens, bw);
+    else
+      hipLaunchKernelGGL((k_encode_blocks<S, D, REV>), dim3(grid), dim3(BS), 0, st, (const S*)data, d.g, d.nblocks,
+                         z, bstage, lens, bw);
+    HIPCHK(hipGetLastError());
+    if ((rc = exclusive_scan(lens, offs, nb1, st)))
+      return rc;
+    hipLaunchKernelGGL(k_clear_edges<0>, dim3(grid_for(nb1, 256)), dim3(256), 0, st, out, offset, (const u64*)offs,
+                       d.nblocks);
+    hipLaunchKernelGGL(k_place_blocks<0>, dim3(grid_for(d.nblocks, 16)), dim3(256), 0, st, (const u64*)bstage, bw,
+                       d.nblocks, out, offset, (const u64*)offs);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(bits_out, offs + d.nblocks, sizeof(u64), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (boffs_out) {
+      *boffs_out = held.p;
+      held.p = nullptr;
+    }
+    return ZFP_HIP_OK;
+  }
+  hipLaunchKernelGGL((k_encode<S, D, ENC_LENGTH, REV>), dim3(grid), dim3(BS), 0, st, (const S*)data, d.g,
+                     d.nblocks, z, out, offset, (const u64*)nullptr, lens);
   HIPCHK(hipGetLastError());
   rc = ws ? exclusive_scan_tmp(lens, offs, nb1, ws->tmp, st) : exclusive_scan(lens, offs, nb1, st);
   if (rc)
@@ -1051,7 +1069,7 @@ int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out
   // a wave's LDS area in the write pass: twice the words 64 average blocks
   // take (64 blocks of b bits take b words), at least 64 and at most 8192
   // (64 KiB); k_encode_waves, four waves per workgroup, takes at most 2048
-  // of them, k_place_blocks, one wave per workgroup, all.  A wave whose
+  // of them.  A wave whose
   // range is longer writes directly, so the size sets the speed, never the
   // stream.  It is taken from the last encode with the same codec
   // parameters; only the first such encode waits for the stream length on
@@ -1084,11 +1102,7 @@ int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out
     hipLaunchKernelGGL(k_prepare_dev, dim3(std::min(grid, 2048u)), dim3(256), 0, st, out, offset,
                        (const u64*)(offs + d.nblocks));
   }
-  if (bstage) {
-    hipLaunchKernelGGL(k_place_blocks<0>, dim3(grid_for(d.nblocks, 64)), dim3(64), (size_t)wcap * 8, st,
-                       (const u64*)bstage, bw, d.nblocks, out, offset, (const u64*)offs, wcap);
-  }
-  else if (stream_order) {
+  if (stream_order) {
     const u32 wc = std::min<u32>(wcap, 2048);
     hipLaunchKernelGGL((k_encode_waves<S, D, REV>), dim3(grid), dim3(BS), (size_t)4 * wc * 8, st, (const S*)data,
                        d.g, d.nblocks, z, out, offset, (const u64*)offs, wc);
@@ -1114,6 +1128,56 @@ int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out
   return ZFP_HIP_OK;
 }
 
+// waits for a decode: the bits it consumed, or ZFP_HIP_ESTALE when a block
+// disagreed with the index (bad)
+inline int decode_result(const Desc& d, const Params& z, bool fixed, const u64* boffs, const u32* bad, u64* bits_out,
+                         hipStream_t st)
+{
+  u64 total = (u64)d.nblocks * z.maxbits;
+  u32 mismatch = 0;
+  if (!fixed)
+    HIPCHK(hipMemcpyAsync(&total, boffs + d.nblocks, sizeof(u64), hipMemcpyDeviceToHost, st));
+  if (bad)
+    HIPCHK(hipMemcpyAsync(&mismatch, bad, sizeof(u32), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  if (mismatch)
+    return ZFP_HIP_ESTALE;
+  *bits_out = total;
+  return ZFP_HIP_OK;
+}
+
+// 4D lossy blocks: k_parse_planes and k_decode_quad over chunks of the field
+// whose plane tables (32 P bytes per block) take at most 256 MiB; smaller
+// chunks when that much is not to be had, ZFP_HIP_ENOMEM when not even 1024
+// blocks fit
+template <typename S>
+int decode_quads(const Desc& d, void* data, const Params& z, const u64* in, u64 nwords, u64 offset,
+                 const u64* boffs, u32* bad, hipStream_t st)
+{
+  constexpr u32 P = Traits<S>::P;
+  u32 groups = std::min((d.nblocks + 63) / 64, (256u << 20) / (P * 4 * 64 * 8)); // 64 blocks each
+  void* p = nullptr;
+  for (;; groups = (groups + 1) / 2) {
+    const int rc = g_stage.get((u64)groups * (P * 4 * 64 * 8 + 64 * 4 + 4), &p);
+    if (rc == ZFP_HIP_OK)
+      break;
+    if (groups <= 16)
+      return rc;
+  }
+  u64* table = (u64*)p;
+  i32* emaxs = (i32*)(table + (u64)groups * P * 4 * 64);
+  u32* low = (u32*)(emaxs + (u64)groups * 64);
+  for (u64 at = 0; at < d.nblocks; at += (u64)groups * 64) {
+    const u32 b0 = (u32)at, nb = std::min(groups * 64, d.nblocks - b0);
+    hipLaunchKernelGGL((k_parse_planes<S>), dim3(grid_for(nb, 64)), dim3(64), 0, st, d.nblocks, b0, nb, z, in, nwords,
+                       offset, boffs, table, low, emaxs, bad);
+    hipLaunchKernelGGL((k_decode_quad<S>), dim3(grid_for(nb, 16)), dim3(64), 0, st, (S*)data, d.g, b0, nb,
+                       (const u64*)table, (const u32*)low, (const i32*)emaxs);
+    HIPCHK(hipGetLastError());
+  }
+  return ZFP_HIP_OK;
+}
+
 template <typename S, int D>
 int launch_decode(const Desc& d, void* data, const Params& z, const u64* in, u64 nwords,
                          u64 offset, const u64* boffs, u64* bits_out, hipStream_t st)
@@ -1122,7 +1186,6 @@ int launch_decode(const Desc& d, void* data, const Params& z, const u64* in, u64
   const unsigned grid = grid_for(d.nblocks, BS);
   const bool rev = is_reversible(z);
   const bool fixed = !rev && z.minbits == z.maxbits;
-  u64 total = 0;
   // a variable-length stream decoded with the caller's index checks every
   // block against it (k_decode's `bad`)
   u32* bad = nullptr;
@@ -1153,6 +1216,17 @@ int launch_decode(const Desc& d, void* data, const Params& z, const u64* in, u64
     else if (rc)
       return rc;
     boffs = (const u64*)lp;
+  }
+  if constexpr (D == 4) {
+    // lossy blocks where the stream has them, one run of bits: parsed lane
+    // by lane, their values decoded over four lanes each
+    if (!rev && (!fixed || !boffs) && block_bits_bound<S, 4, false>(z) <= 8 * (PARSE_WORDS - 4)) {
+      int rc = decode_quads<S>(d, data, z, in, nwords, offset, boffs, bad, st);
+      if (rc == ZFP_HIP_OK)
+        return decode_result(d, z, fixed, boffs, bad, bits_out, st);
+      if (rc != ZFP_HIP_ENOMEM)
+        return rc;
+    }
   }
   // fixed rate: stage blocks through LDS when a workgroup's slots fit in
   // 64 KiB (an odd slot stride spreads the lanes over the LDS banks)
@@ -1213,18 +1287,7 @@ int launch_decode(const Desc& d, void* data, const Params& z, const u64* in, u64
                        nwords, offset, boffs, 0u, (u32*)nullptr, (u32*)nullptr, bad);
   }
   HIPCHK(hipGetLastError());
-  u32 mismatch = 0;
-  if (fixed)
-    total = (u64)d.nblocks * z.maxbits;
-  else
-    HIPCHK(hipMemcpyAsync(&total, boffs + d.nblocks, sizeof(u64), hipMemcpyDeviceToHost, st));
-  if (bad)
-    HIPCHK(hipMemcpyAsync(&mismatch, bad, sizeof(u32), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  if (mismatch)
-    return ZFP_HIP_ESTALE;
-  *bits_out = total;
-  return ZFP_HIP_OK;
+  return decode_result(d, z, fixed, boffs, bad, bits_out, st);
 }
 
 template <int D>
