@@ -1,0 +1,139 @@
+"""Variable-length float streams without an index, whose block starts come from
+guessed starts (k_sync_*, codec_sync.h).  The guesses decide how many rounds
+that takes and never the result, so each field here makes them fail in its own
+way: exponents that neighbours do not share, exponents that few blocks have,
+blocks of zeros in long runs and alone, arbitrary words in the stream's place.
+The codec is exact: every value equals the oracle's, the bits consumed too."""
+import zlib
+
+import numpy as np
+import pytest
+
+from test_device_code_on_host import lib
+from zfptest import (NP_OF_TYPE, T_DOUBLE, T_FLOAT, field_args, make_layout, oracle_compress, oracle_decompress,
+                     smooth_field, stream_params_accuracy, stream_params_precision, u64p)
+
+TYPES = {"f32": T_FLOAT, "f64": T_DOUBLE}
+# blocks: 1, a segment or two, many segments at the edges of a wave's 64
+SHAPES = {"one": [4, 3], "few": [70, 9], "1d": [9001], "2d": [517, 260], "3d": [65, 50, 43], "2d_large": [1501, 1100]}
+MODES = {
+    "prec5": lambda t: stream_params_precision(5),
+    "prec28": lambda t: stream_params_precision(28),
+    "prec64": lambda t: stream_params_precision(64),
+    "acc1e-3": lambda t: stream_params_accuracy(1e-3),
+    "padded": lambda t: (200, 16658, 20, -1074),   # blocks of 200 bits at least
+    "cut": lambda t: (1, 150, 30, -1074),          # blocks of 150 bits at most
+}
+
+
+def field(n, ztype, content):
+    rng = np.random.default_rng(zlib.crc32(f"{n}/{ztype}/{content}".encode()))
+    a = smooth_field(n, ztype, seed=len(content)).astype(np.float64)
+    if content == "scales":
+        # every value on a scale of its own: neighbouring exponents far apart
+        a = np.ldexp(a, rng.integers(-40, 40, a.size))
+    elif content == "corner":
+        a[: a.size // 50] *= 2.0 ** -30
+    elif content == "zeros":
+        a[rng.random(a.size) < 0.999] = 0.0
+        a[a.size // 3: a.size // 2] = 0.0
+    return a.astype(NP_OF_TYPE[ztype])
+
+
+def decode(words, n, ztype, params, offset):
+    import torch
+
+    import zfp_amd as Z
+    w = torch.from_numpy(words.view(np.int64)).cuda()
+    out = torch.zeros(int(np.prod(n)), dtype=torch.float32 if ztype == T_FLOAT else torch.float64, device="cuda")
+    Z.hip_lib().zfp_hip_index_clear()
+    bits = Z.decode(ztype, n, None, out.data_ptr(), params, w.data_ptr(), offset=offset, nwords=w.numel())
+    return bits, out.cpu().numpy()
+
+
+def expected(words, n, ztype, params, offset):
+    want = np.zeros(int(np.prod(n)), NP_OF_TYPE[ztype])
+    base, off, s = make_layout(want, n, "as_is")
+    padded = np.concatenate([words, np.zeros(64, np.uint64)]) # the oracle's reads past the end
+    oracle_decompress(padded, base, off, n, s, ztype, params, offset)
+    return base
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("content", ["smooth", "scales", "corner", "zeros"])
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("shape", [k for k in SHAPES if k != "2d_large"])
+def test_streams_without_index(shape, tname, mode, content):
+    n, ztype = SHAPES[shape], TYPES[tname]
+    params = MODES[mode](ztype)
+    a = field(n, ztype, content)
+    base, off, s = make_layout(a, n, "as_is")
+    words, bits = oracle_compress(base, off, n, s, ztype, params)[:2]
+    words = np.asarray(words)[: (bits + 63) // 64].copy()
+    got_bits, got = decode(words, n, ztype, params, 0)
+    assert got_bits == bits
+    assert np.array_equal(got.view(np.uint8), expected(words, n, ztype, params, 0).view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tail", ["zeros", "garbage"])
+@pytest.mark.parametrize("offset", [1, 77, 128])
+@pytest.mark.parametrize("tname", list(TYPES))
+def test_stream_inside_a_buffer(tname, offset, tail):
+    """The stream at a bit offset, and its buffer longer than it is."""
+    n, ztype = SHAPES["2d_large"], TYPES[tname]
+    params = MODES["prec28"](ztype)
+    a = field(n, ztype, "smooth")
+    base, off, s = make_layout(a, n, "as_is")
+    words, bits = oracle_compress(base, off, n, s, ztype, params, offset)[:2]
+    used = (offset + bits + 63) // 64
+    rng = np.random.default_rng(offset)
+    extra = np.zeros(used // 2, np.uint64) if tail == "zeros" else rng.integers(0, 2 ** 64, used // 2, np.uint64)
+    buf = np.concatenate([np.asarray(words)[:used], extra])
+    got_bits, got = decode(buf, n, ztype, params, offset)
+    assert got_bits == bits
+    assert np.array_equal(got.view(np.uint8), expected(buf, n, ztype, params, offset).view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ones", [0.02, 0.5, 0.95])
+@pytest.mark.parametrize("mode", ["prec5", "prec28", "padded", "cut"])
+@pytest.mark.parametrize("tname", list(TYPES))
+@pytest.mark.parametrize("shape", ["1d", "2d", "3d"])
+def test_arbitrary_words(shape, tname, mode, ones):
+    """Any bits are a stream; words enough for every block at its longest."""
+    n, ztype = SHAPES[shape], TYPES[tname]
+    params = MODES[mode](ztype)
+    rng = np.random.default_rng(zlib.crc32(f"{shape}/{tname}/{mode}/{ones}".encode()))
+    blocks = int(np.prod([(v + 3) // 4 for v in n]))
+    longest = max(params[0], min(params[1], 12 + 4 ** len(n) * (params[2] + 1)))
+    words = np.packbits(rng.random((blocks * longest // 64 + 1, 64)) < ones, axis=1, bitorder="little")
+    words = words.view(np.uint64).reshape(-1).copy()
+    got_bits, got = decode(words, n, ztype, params, 0)
+    want = np.zeros(int(np.prod(n)), NP_OF_TYPE[ztype])
+    nn, ss = field_args(n, None)
+    bits = lib().hostcodec_decompress(ztype, nn, ss, want.ctypes.data, *params, words.ctypes.data_as(u64p),
+                                      words.size, 0)
+    assert got_bits == bits
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.gpu
+def test_stream_of_several_chunks():
+    """More than 2^31 bits: a second chunk starts at the first one's exit."""
+    import torch
+
+    import zfp_amd as Z
+    n, params = [420, 400, 400], stream_params_precision(52)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.rand(n[2] * n[1] * n[0], dtype=torch.float64, device="cuda", generator=g)
+    w = torch.zeros(Z.max_stream_words(T_DOUBLE, n, params), dtype=torch.int64, device="cuda")
+    bits = Z.encode(T_DOUBLE, n, None, a.data_ptr(), params, w.data_ptr())
+    assert bits > 1.5 * 2 ** 31
+    used = (bits + 63) // 64
+    indexed, parsed = torch.zeros_like(a), torch.zeros_like(a)
+    assert Z.decode(T_DOUBLE, n, None, indexed.data_ptr(), params, w.data_ptr(), nwords=used) == bits
+    Z.hip_lib().zfp_hip_index_clear()
+    assert Z.decode(T_DOUBLE, n, None, parsed.data_ptr(), params, w.data_ptr(), nwords=used) == bits
+    assert torch.equal(indexed, parsed)

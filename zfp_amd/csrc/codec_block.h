@@ -114,9 +114,8 @@ __device__ __forceinline__ void decode_half(PlaneDecoder<N>& pd, R& r, PlaneVec&
 // when the block goes on below plane 32; such a block's coefficients lack
 // their low half and it has to be decoded again in full.  Leaving the low
 // half out frees the registers that hold it.
-template <int N, int P, typename UInt, bool STORE, bool HI_ONLY = false, typename R = BitReader>
-__device__ __forceinline__ u32 decode_planes(R& r, UInt* u, u32 maxbits, u32 maxprec,
-                                             bool* more = nullptr)
+template <int N, int P, typename UInt, bool HI_ONLY, typename R>
+__device__ __forceinline__ u32 decode_plane_values(R& r, UInt* u, u32 maxbits, u32 maxprec, bool* more)
 {
   static_assert(!HI_ONLY || P == 64, "HI_ONLY splits 64-bit coefficients");
   PlaneDecoder<N> pd;
@@ -125,11 +124,10 @@ __device__ __forceinline__ u32 decode_planes(R& r, UInt* u, u32 maxbits, u32 max
   PlaneVec lo, hi;
   if constexpr (P == 64) {
     decode_half<N>(pd, r, lo, hi, 32);
-    if (STORE)
-      coeffs_half<N>(lo, hi, w);
+    coeffs_half<N>(lo, hi, w);
 #pragma unroll
     for (int i = 0; i < N; i++)
-      u[i] = STORE ? (UInt)w[i] << (P / 2) : 0;
+      u[i] = (UInt)w[i] << (P / 2);
     if constexpr (HI_ONLY) {
       *more = pd.wants(31);
       return pd.used();
@@ -142,14 +140,23 @@ __device__ __forceinline__ u32 decode_planes(R& r, UInt* u, u32 maxbits, u32 max
   }
   if (wave_any(pd.wants(31))) {
     decode_half<N>(pd, r, lo, hi, 0);
-    if (STORE) {
-      coeffs_half<N>(lo, hi, w);
+    coeffs_half<N>(lo, hi, w);
 #pragma unroll
-      for (int i = 0; i < N; i++)
-        u[i] |= (UInt)w[i];
-    }
+    for (int i = 0; i < N; i++)
+      u[i] |= (UInt)w[i];
   }
   return pd.used();
+}
+
+// Without STORE only the length is wanted: u is left unset and the reader
+// anywhere.
+template <int N, int P, typename UInt, bool STORE, bool HI_ONLY = false, typename R = BitReader>
+__device__ __forceinline__ u32 decode_planes(R& r, UInt* u, u32 maxbits, u32 maxprec, bool* more = nullptr)
+{
+  if constexpr (STORE)
+    return decode_plane_values<N, P, UInt, HI_ONLY>(r, u, maxbits, maxprec, more);
+  else
+    return planes_length<N>(r, P, maxbits, maxprec);
 }
 
 // ---------------------------------------------------------------------------

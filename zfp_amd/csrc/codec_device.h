@@ -1249,6 +1249,113 @@ struct PlaneDecoder {
 };
 
 // --------------------------------------------------------------------------
+// Lengths of planes without their values, for finding where blocks start.
+// A lane cannot know its block's length before it has gone through its
+// planes, and a wave that takes a trip per new coefficient takes the most
+// trips of any lane for every plane.  Here a plane's group tests are one
+// straight run of instructions: of the one-bits, the 1st, 3rd, ... are tests
+// and the 2nd, 4th, ... the coefficients they find, told apart by a prefix
+// parity, and the plane ends at the first 0 after one of the latter.  Once
+// every coefficient is significant the rest of the length is a product.
+// --------------------------------------------------------------------------
+
+// bit i: the parity of bits 0 .. i
+ZH_INLINE u32 prefix_parity(u32 x)
+{
+  x ^= x << 1;
+  x ^= x << 2;
+  x ^= x << 4;
+  x ^= x << 8;
+  x ^= x << 16;
+  return x;
+}
+ZH_INLINE u64 prefix_parity(u64 x)
+{
+  const u32 lo = prefix_parity((u32)x);
+  const u32 hi = prefix_parity((u32)(x >> 32)) ^ (u32)((i32)lo >> 31);
+  return (u64)hi << 32 | lo;
+}
+
+// position of the k-th (from 0) one-bit of x, which has more than k of them
+ZH_INLINE u32 select_one(u32 x, u32 k)
+{
+  u32 p = 0;
+#pragma unroll
+  for (u32 h = 16; h; h >>= 1) {
+    const u32 c = (u32)__builtin_popcount(x & ((1u << h) - 1));
+    const bool up = k >= c;
+    k -= up ? c : 0u;
+    x >>= up ? h : 0u;
+    p += up ? h : 0u;
+  }
+  return p;
+}
+ZH_INLINE u32 select_one(u64 x, u32 k)
+{
+  const u32 c = (u32)__builtin_popcount((u32)x);
+  const bool up = k >= c;
+  return (up ? 32u : 0u) + select_one(up ? (u32)(x >> 32) : (u32)x, up ? k - c : k);
+}
+
+// Bits of the planes of N <= 64 coefficients at the reader (P - 1 down, as
+// PlaneDecoder counts them).  The planes are read without the budget, which
+// cuts the sum: a budgeted code is a prefix of the unbudgeted one.  Leaves
+// the reader anywhere.
+template <int N, typename R>
+ZH_INLINE u32 planes_length(R& r, u32 P, u32 maxbits, u32 maxprec)
+{
+  // a plane of N <= 16 coefficients ends within 32 bits of its first test
+  typedef typename std::conditional<N <= 16, u32, u64>::type W;
+  constexpr u32 WBITS = 8 * sizeof(W);
+  const u32 limit = budget_binds(maxbits, maxprec, N) ? maxbits : 0xffffffffu;
+  u32 planes = umin(P, maxprec), rem = N, pos = 0;
+#pragma unroll 1
+  for (; planes && rem && pos < limit; planes--) {
+    const u32 n = N - rem;
+    u32 len; // the plane's bits
+    W w;
+    if constexpr (N <= 16) {
+      w = (W)(r.peek64() >> n);
+      len = n;
+    }
+    else {
+      r.skip(n);
+      w = r.peek64();
+      len = 0;
+      pos += n;
+    }
+    W run = 0; // all ones when the window starts within a run
+    for (;;) {
+      const W odd = prefix_parity(w) ^ run;
+      const W tests = w & odd;
+      const u32 end = umin(first_one((W)(~w & (((w & ~odd) << 1) | (~run & 1)))), WBITS);
+      // coefficients found before the end: its bits but the tests
+      const u32 c = end - (u32)__builtin_popcountll(tests & (W)lowmask(end));
+      if (c >= rem) {
+        // the last coefficient's one-bit is implied
+        len += select_one((W)~tests, rem - 1);
+        rem = 0;
+        break;
+      }
+      rem -= c;
+      if (N <= 16 || end < WBITS) {
+        len += end + 1;
+        break;
+      }
+      r.skip(64);
+      pos += 64;
+      w = (W)r.peek64();
+      run = (W)0 - (odd >> (WBITS - 1));
+    }
+    r.skip(len);
+    pos += len;
+  }
+  if (pos < limit && !rem)
+    pos += planes * N;
+  return umin(pos, limit);
+}
+
+// --------------------------------------------------------------------------
 // 4D blocks (256 coefficients): planes are four 64-bit words; the coder
 // follows encode_many_ints / decode_many_ints (encode.c:134-176,
 // decode.c:133-184), which produce the same code as the N <= 64 variants.

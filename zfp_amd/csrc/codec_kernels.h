@@ -849,6 +849,12 @@ int chain_parse(const Desc& d, const Params& z, const u64* in, u64 nwords, u64 o
   return 0;
 }
 
+} // namespace zfphip
+
+#include "codec_sync.h"
+
+namespace zfphip {
+
 template <typename S, int D, bool REV>
 int launch_encode_var(const Desc& d, const void* data, const Params& z, u64* out, u64 offset, u64* bits_out,
                       hipStream_t st, u64** boffs_out, const Workspace* ws);
@@ -1198,12 +1204,19 @@ int launch_decode(const Desc& d, void* data, const Params& z, const u64* in, u64
     HIPCHK(hipMemsetAsync(bad, 0, sizeof(u32), st));
   }
   if (!fixed && !boffs) {
-    // no index: recover block offsets by a sequential parse
+    // no index: block starts from guesses by their exponents where blocks
+    // have one, else (or where those do not settle) by chains from
+    // arbitrary bits, else by a sequential parse
     void* lp;
     int rc = g_lens.get(((u64)d.nblocks + 1) * sizeof(u64), &lp);
     if (rc)
       return rc;
-    rc = chain_parse<S, D>(d, z, in, nwords, offset, (u64*)lp, st);
+    rc = CHAIN_FALLBACK;
+    if constexpr (Traits<S>::FLOAT && D < 4)
+      if (!rev)
+        rc = sync_parse<S, D>(d, z, in, nwords, offset, (u64*)lp, st);
+    if (rc == CHAIN_FALLBACK)
+      rc = chain_parse<S, D>(d, z, in, nwords, offset, (u64*)lp, st);
     if (rc == CHAIN_FALLBACK) {
       if (rev)
         hipLaunchKernelGGL((k_parse<S, D, true>), dim3(1), dim3(64), 0, st, d.g, d.nblocks, z, in, nwords,

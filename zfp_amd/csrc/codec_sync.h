@@ -1,0 +1,628 @@
+// codec_sync.h -- block starts of a variable-length float stream that arrives
+// without an index, from guessed starts that are then proven.
+//
+// The stream's bits are cut into segments of about SYNC_BLOCKS blocks, one
+// lane each.  A segment's lane can only follow block lengths once it knows
+// where some block starts, and a chain of lengths from an arbitrary bit meets
+// the true one only after about as many blocks as a block has bits.  A block
+// of floats does, however, open with its exponent, which is close to its
+// neighbours': a bit from which block after block opens with a 1 and an
+// exponent within SYNC_NEAR of the one before is a block start but for a
+// chance of (7/512)^hops.
+//
+//   k_sync_sample     waves search some segments for chains of any exponent
+//   k_sync_range      and count the exponents met, which gives a range of
+//                     exponents worth trying;
+//   k_sync_guess      a lane group per segment tries the bits that open with
+//                     a 1 and an exponent in that range, the first that
+//                     starts a chain being the guess;
+//   k_sync_retry      segments without a guess are searched like the samples
+//                     when they are many;
+//   k_sync_walk       one lane per segment follows the chain from its guess
+//                     to its exit, the first position at or past the
+//                     segment's end, setting a bit per position in `marks`;
+//                     then rounds, in which a lane whose start is not its
+//                     predecessor's exit t moves its start to t: the chain
+//                     from t meets its old one at a marked bit, where the
+//                     old marks and exit stand, or replaces it;
+//   k_marks_*         block numbers by counting marks, and the offsets.
+//
+// When every segment's start is its predecessor's exit, and the first start
+// is the stream's, every mark is by induction a block start: guesses decide
+// how many rounds that takes (two or three), never the result.
+//
+// The walk is bound by the latency of the plane loop's dependent instructions
+// (a plane is one straight run of them, planes_length), so segments are short
+// enough for four or more waves per SIMD.  Against chains from arbitrary bits
+// in segments of 32 Kibit (chain_lane), which need a round for every segment
+// that chains do not meet in, whole decodes of f32 fields: 8191 x 8193 at
+// precision 16 13.7 -> 1.20 ms, at precision 28 37.6 -> 1.75 ms; 401 x 402 x
+// 403 at precision 28 207 -> 2.0 ms; 300 x 301 within 1e-3 6.4 -> 0.25 ms.
+// chain_lane stays for blocks that open with no exponent of their own
+// (integers, reversible ones), for 4D blocks, and for fields whose exponents
+// are no guide.
+#pragma once
+
+namespace zfphip {
+
+constexpr u32 SYNC_WORDS = 16;    // words of the stream a lane stages at a time
+constexpr u32 SYNC_SLOT = 2 * SYNC_WORDS + 1; // 32-bit words of its slot, odd to spread the lanes over the banks
+constexpr int SYNC_NEAR = 3;      // exponents of neighbouring blocks, at most this far apart
+constexpr u32 SYNC_SAMPLES = 256;
+constexpr u64 SYNC_NONE = ~0ull;  // a segment's start or exit that is not known yet
+constexpr u32 SYNC_ROUNDS = 3;    // rounds between looks from the host
+constexpr u32 SYNC_LOOKS = 16;
+
+// what the host looks at, on the device
+struct SyncState {
+  u32 seen[2048];              // how often each exponent was sampled
+  u32 lo, hi;                  // the exponents to look for
+  u32 missed;                  // segments without a guess
+  u32 open[SYNC_ROUNDS];       // per round, the first segment that did not start at its predecessor's exit (~0: none)
+  u64 total, exit;             // marks in the chunk, its last segment's exit
+};
+
+struct SyncArgs {
+  Params z;
+  const u64* in;
+  u64 nwords, offset, span;    // as in ChainArgs
+  u64 at, bits, L;             // the chunk's first bit, its bits, and bits per segment (64 k)
+  u64 entry;                   // the first block start at or past `at`
+  u32 P, samples, step;        // segments, samples and their distance
+  u32 window, hops, need;      // bits a guess may look at, hops it has to hold; bits to have staged per block
+  const u64* start_prev;       // the segments' starts and exits before and
+  const u64* exit_prev;        // after a round
+  u64* start_new;
+  u64* exit_new;
+  u64* marks;                  // bit p: a chain position at chunk bit p; whole tiles of 4096
+  SyncState* state;
+
+  __device__ __forceinline__ u64 seg_end(u32 i) const { return at + (i + 1 == P ? bits : (u64)(i + 1) * L); }
+};
+
+// Reads from SYNC_WORDS words of the stream that the lane staged in its slot
+// of LDS, all loads in flight at once, and past them from memory.  A reader
+// that loads word by word waits out the memory's latency at nearly every
+// plane, since at nearly every plane some lane of the wave needs its next
+// word.
+struct StageReader {
+  const u64* in;
+  u64 nwords, word0; // the slot's first word in the stream
+  u32* slot;
+  u32 pos;           // bits from word0
+
+  ZH_INLINE void stage(u64 bit)
+  {
+    word0 = bit >> 6;
+    pos = (u32)(bit & 63);
+    u64 v[SYNC_WORDS];
+#pragma unroll
+    for (u32 k = 0; k < SYNC_WORDS; k++)
+      v[k] = in[word0 + k < nwords ? word0 + k : nwords - 1];
+#pragma unroll
+    for (u32 k = 0; k < SYNC_WORDS; k++) {
+      const u64 x = word0 + k < nwords ? v[k] : 0ull;
+      slot[2 * k] = (u32)x;
+      slot[2 * k + 1] = (u32)(x >> 32);
+    }
+  }
+  // to stream bit `bit` (at or past word0), the slot holding n bits from there
+  ZH_INLINE void seek(u64 bit, u32 n)
+  {
+    pos = (u32)(bit - (word0 << 6));
+    // all lanes together, so that the wave waits for memory once
+    if (wave_any(pos + n > 64 * SYNC_WORDS))
+      stage(bit);
+  }
+  ZH_INLINE u64 load(u64 i) const { return i < nwords ? in[i] : 0ull; }
+  ZH_INLINE u64 peek64() const
+  {
+    const u32 i = pos >> 5;
+    if (i + 2 < 2 * SYNC_WORDS)
+      return (u64)funnel32(slot[i + 1], slot[i], pos) | (u64)funnel32(slot[i + 2], slot[i + 1], pos) << 32;
+    const u64 w = word0 + (pos >> 6);
+    return (load(w) >> (pos & 63)) | ((load(w + 1) << 1) << (63 - (pos & 63)));
+  }
+  ZH_INLINE u64 peek(u32 n) const { return peek64() & lowmask(n); }
+  ZH_INLINE void skip(u32 n) { pos += n; }
+  ZH_INLINE u64 read(u32 n) { u64 v = peek(n); skip(n); return v; }
+};
+
+// the length, at least 1, of the block at the reader
+template <typename S, int D>
+ZH_INLINE u32 sync_block(StageReader& r, const Params& z)
+{
+  const Geom g{};
+  const u32 bc[4] = {0, 0, 0, 0};
+  const u32 len = decode_block<S, D, false>(r, (S*)nullptr, g, bc, z);
+  return len ? len : 1;
+}
+
+// the exponent a block opens with, or -1 when v opens with a 0 or with an
+// exponent that codes no plane
+template <typename S, int D>
+ZH_INLINE int sync_exponent(u64 v, const Params& z)
+{
+  typedef Traits<S> T;
+  const int e = (int)(v >> 1) & ((1 << T::EBITS) - 1);
+  return (v & 1) && plane_count(e - T::EBIAS, z.maxprec, z.minexp, D) ? e : -1;
+}
+
+// whether `hops` blocks from stream bit p on are followed by a block of a
+// near exponent each (blocks of zeros, single 0 bits, skipped); lo, hi: the
+// exponents met
+template <typename S, int D>
+ZH_INLINE bool sync_hops(const SyncArgs& a, u32* slot, u64 p, u32 hops, int& lo, int& hi)
+{
+  StageReader r{a.in, a.nwords, 0, slot, 0};
+  r.stage(a.offset + p);
+  int e = sync_exponent<S, D>(r.peek64(), a.z);
+  lo = hi = e;
+  bool ok = e >= 0;
+  for (u32 h = 0; h < hops && ok; h++) {
+    p += sync_block<S, D>(r, a.z);
+    r.seek(a.offset + p, h + 1 < hops ? a.need : 64);
+    u64 v = r.peek64();
+    if (!(v & 1)) {
+      p += a.z.minbits > 1 ? a.z.minbits : umin(ctz64z(v), 63u);
+      r.seek(a.offset + p, h + 1 < hops ? a.need : 64);
+      v = r.peek64();
+    }
+    if (p >= a.span)
+      return h > 0;
+    const int f = sync_exponent<S, D>(v, a.z);
+    ok = f >= 0 && f - e <= SYNC_NEAR && e - f <= SYNC_NEAR;
+    e = f;
+    lo = f < lo ? f : lo;
+    hi = f > hi ? f : hi;
+  }
+  return ok;
+}
+
+// The first of bits [base, lim) from which a chain holds, whatever exponent
+// it opens with, searched by a wave 64 candidates at a time; SYNC_NONE when
+// there is none.  lo, hi: the exponents met, in the lane that has `mine`.
+template <typename S, int D>
+ZH_INLINE u64 sync_search(const SyncArgs& a, u32* queue, u32* slots, u64 base, u64 lim, int& lo, int& hi, bool& mine)
+{
+  const u32 lane = threadIdx.x & 63u;
+  u32 cnt = 0;
+  for (u64 p = base;;) {
+    while (cnt < 64 && p < lim) {
+      const u64 q = p + lane;
+      bool ok = false;
+      if (q < lim) {
+        const u64 bit = a.offset + q, w = bit >> 6; // w < nwords, as q < span
+        const u32 s = (u32)(bit & 63);
+        const u64 v = (a.in[w] >> s) | ((w + 1 < a.nwords ? a.in[w + 1] << 1 : 0ull) << (63 - s));
+        ok = sync_exponent<S, D>(v, a.z) >= 0;
+      }
+      const u64 m = __ballot(ok);
+      if (ok)
+        queue[cnt + (u32)__builtin_popcountll(m & lowmask(lane))] = (u32)(q - base);
+      cnt += (u32)__builtin_popcountll(m);
+      p += 64;
+    }
+    if (!cnt)
+      return SYNC_NONE;
+    wave_lds_sync();
+    const u32 n = umin(cnt, 64u), later = queue[lane + 64];
+    bool good = false;
+    if (lane < n)
+      good = sync_hops<S, D>(a, slots + lane * SYNC_SLOT, base + queue[lane], a.hops + 1, lo, hi);
+    const u64 m = __ballot(good);
+    if (m) {
+      mine = lane == ctz64(m);
+      return base + queue[ctz64(m)];
+    }
+    wave_lds_sync();
+    queue[lane] = later; // what was queued past the 64 tried
+    cnt -= n;
+  }
+}
+
+// Samples segments i * step: four waves search a quarter of the segment's
+// window each, and the exponents of the chains they find are counted.
+template <typename S, int D>
+__global__ void __launch_bounds__(256)
+k_sync_sample(SyncArgs a)
+{
+  __shared__ u32 queue[4][128];
+  __shared__ u32 slots[256 * SYNC_SLOT];
+  const u32 i = blockIdx.x * a.step, wave = threadIdx.x >> 6;
+  const u64 end = a.at + (u64)i * a.L + a.window;
+  const u64 base = end - a.window + (u64)wave * (a.window / 4 + 1);
+  const u64 lim = std::min(std::min(base + a.window / 4 + 1, end), a.seg_end(i));
+  int lo = 0, hi = -1;
+  bool mine = false;
+  if (base < lim)
+    sync_search<S, D>(a, queue[wave], slots + wave * 64 * SYNC_SLOT, base, lim, lo, hi, mine);
+  if (mine)
+    for (int e = lo; e <= hi; e++)
+      atomicAdd(&a.state->seen[e], 1u);
+}
+
+// Of the 32 stream bits from bit q on, those that open with a 1 and an
+// exponent in [lo, hi], compared for all 32 at once: bit by bit of the
+// exponent, from the lowest, the majority of the bit, the comparison so far
+// and the bound's bit decides.
+template <typename S>
+ZH_INLINE u32 sync_matches(const SyncArgs& a, u64 q, u32 lo, u32 hi)
+{
+  const u64 bit = a.offset + q, w = bit >> 6; // w < nwords, as q < span
+  const u32 s = (u32)(bit & 63);
+  const u64 v = (a.in[w] >> s) | ((w + 1 < a.nwords ? a.in[w + 1] << 1 : 0ull) << (63 - s));
+  u32 ge = ~0u, le = ~0u;
+#pragma unroll
+  for (int j = 0; j < Traits<S>::EBITS; j++) {
+    const u32 b = (u32)(v >> (j + 1));
+    const u32 nlo = (lo >> j & 1u) - 1u, mhi = 0u - (hi >> j & 1u); // ~lo's and hi's bit j, as masks
+    ge = (b & ge) | (nlo & (b | ge));
+    le = (~b & le) | (mhi & (~b | le));
+  }
+  return (u32)v & ge & le;
+}
+
+// The exponents to look for: the range of those whose count, with their
+// neighbours', is a 16th of the largest such count.  (One wave; chance finds
+// are of any exponent.)
+template <typename S>
+__global__ void __launch_bounds__(64)
+k_sync_range(SyncArgs a)
+{
+  constexpr u32 E = 1u << Traits<S>::EBITS;
+  const u32* seen = a.state->seen;
+  auto count = [&](u32 k) { return seen[k] + (k ? seen[k - 1] : 0u) + (k + 1 < E ? seen[k + 1] : 0u); };
+  u32 most = 0;
+  for (u32 k = threadIdx.x; k < E; k += 64)
+    most = std::max(most, count(k));
+  for (u32 d = 32; d; d >>= 1)
+    most = std::max(most, (u32)__shfl_xor(most, d, 64));
+  u32 lo = E, hi = 0;
+  for (u32 k = threadIdx.x; k < E; k += 64) {
+    const u32 c = count(k);
+    const u64 m = __ballot(c && 16 * c >= most);
+    if (m) {
+      const u32 k0 = k - threadIdx.x;
+      lo = umin(lo, k0 + ctz64(m));
+      hi = k0 + 63u - (u32)__builtin_clzll(m);
+    }
+  }
+  if (threadIdx.x == 0) {
+    a.state->lo = lo;
+    a.state->hi = hi;
+  }
+}
+
+// The start of every segment, G lanes each, and its marks zeroed: the first
+// candidate that holds, SYNC_NONE when none does.  Each lane tries the
+// candidates of its own 32-bit pieces of the window, in order, as long as
+// they lie before the best of the group's.
+template <typename S, int D, int G>
+__global__ void __launch_bounds__(64)
+k_sync_guess(SyncArgs a)
+{
+  __shared__ u32 slots[64 * SYNC_SLOT];
+  const u32 lane = threadIdx.x, grp = lane / G, gl = lane % G;
+  const u32 i = blockIdx.x * (64 / G) + grp;
+  const bool valid = i < a.P;
+  const u64 base = a.at + (u64)(valid ? i : 0) * a.L, end = a.seg_end(valid ? i : 0);
+  if (valid) {
+    // the last segment clears up to the end of its tile
+    const u64 w1 = i + 1 == a.P ? (a.bits + 4095) / 4096 * 64 : (end - a.at) / 64;
+    for (u64 w = (base - a.at) / 64 + gl; w < w1; w += G)
+      a.marks[w] = 0;
+  }
+  const u32 lo = a.state->lo, hi = a.state->hi;
+  // the bits to look at: none in the first segment
+  const u32 window = valid && i ? (u32)std::min<u64>(a.window, end - base) : 0u;
+  u32 best = window, p = 32 * gl, m = 0;
+  bool done = false;
+#pragma unroll 1
+  while (wave_any(!done)) {
+    while (!m && p < best) {
+      m = sync_matches<S>(a, base + p, lo, hi);
+      p += 32 * G;
+    }
+    const u32 q = p - 32 * G + (m ? ctz64(m) : 0u);
+    u32 mine = best;
+    if (m && q < best) {
+      int l, h;
+      m &= m - 1;
+      if (sync_hops<S, D>(a, slots + lane * SYNC_SLOT, base + q, a.hops, l, h))
+        mine = q;
+    }
+    else
+      m = 0;
+#pragma unroll
+    for (u32 d = 1; d < (u32)G; d <<= 1)
+      mine = umin(mine, (u32)__shfl_xor(mine, d, 64));
+    best = mine;
+    done = !m && p >= best;
+  }
+  if (valid && gl == 0)
+    a.start_new[i] = !i ? a.entry : best < window ? base + best : SYNC_NONE;
+  const u64 none = __ballot(valid && i && gl == 0 && best >= window);
+  if (none && lane == 0)
+    atomicAdd(&a.state->missed, (u32)__builtin_popcountll(none));
+}
+
+// When guesses miss in more than one segment of 128 (exponents that the
+// samples met too seldom), those segments are searched whatever the
+// exponent; fewer are left to the rounds, and when most miss, exponents say
+// nothing here.
+template <typename S, int D>
+__global__ void __launch_bounds__(64)
+k_sync_retry(SyncArgs a)
+{
+  __shared__ u32 queue[128];
+  __shared__ u32 slots[64 * SYNC_SLOT];
+  if (a.state->missed <= a.P / 128 + 2 || a.state->missed > a.P / 2)
+    return;
+  for (u32 i = blockIdx.x; i < a.P; i += gridDim.x) {
+    if (a.start_new[i] != SYNC_NONE)
+      continue;
+    const u64 base = a.at + (u64)i * a.L;
+    int lo, hi;
+    bool mine;
+    const u64 found = sync_search<S, D>(a, queue, slots, base, std::min(base + a.window, a.seg_end(i)), lo, hi, mine);
+    if (threadIdx.x == 0)
+      a.start_new[i] = found;
+    wave_lds_sync();
+  }
+}
+
+// round 0: every lane follows its chain from its start.  Later rounds (round
+// r: a.state->open[r - 1]): a lane whose start is not its predecessor's exit
+// takes that exit for its start, unless the predecessor's own start is not
+// its predecessor's exit: a wrong chain would then run on through segments
+// that had started right.  (The first such lane always moves.)
+template <typename S, int D>
+__global__ void __launch_bounds__(64)
+k_sync_walk(SyncArgs a, u32 round)
+{
+  __shared__ u32 slots[64 * SYNC_SLOT];
+  const u32 i = blockIdx.x * 64 + threadIdx.x;
+  bool open = false;
+  if (i < a.P) {
+    const u64 begin = (u64)i * a.L, end = a.seg_end(i) - a.at; // in the chunk, as `pos` and the marks
+    const u64 s = a.start_prev[i];
+    u64 t = s, out = round ? a.exit_prev[i] : s;
+    if (round && i) {
+      const u64 e = a.exit_prev[i - 1];
+      open = s != e || e == SYNC_NONE;
+      if (open && e != SYNC_NONE && (i == 1 || a.start_prev[i - 1] == a.exit_prev[i - 2]))
+        t = e;
+    }
+    if (round ? s != t : s != SYNC_NONE) {
+      const bool runs = a.z.minbits <= 1;
+      u64 pos = t - a.at;
+      u64 cur = pos < end ? pos >> 6 : end >> 6;
+      u64 word = 0, old = 0;
+      bool met = false;
+      if (round)
+        for (u64 w = begin >> 6; w < cur; w++)
+          a.marks[w] = 0;
+      if (pos < end) {
+        old = a.marks[cur];
+        StageReader r{a.in, a.nwords, 0, slots + threadIdx.x * SYNC_SLOT, 0};
+        r.stage(a.offset + t);
+#pragma unroll 1
+        while (pos < end) {
+          if (pos >> 6 != cur) {
+            a.marks[cur] = word;
+            for (cur++; cur < pos >> 6; cur++)
+              a.marks[cur] = 0;
+            word = 0;
+            old = round ? a.marks[cur] : 0ull;
+          }
+          r.seek(a.offset + a.at + pos, a.need);
+          const u32 b = (u32)(pos & 63);
+          u32 n = 1; // blocks in this step: a run of zero bits is a run of blocks
+          bool coded = true;
+          if (runs) {
+            const u64 v = r.peek64();
+            if (!(v & 1)) {
+              coded = false;
+              n = umin(ctz64z(v), 64u - b);
+              n = end - pos < n ? (u32)(end - pos) : n;
+            }
+          }
+          const u64 hit = (old >> b) & lowmask(n);
+          if (hit) {
+            // the old chain from here on
+            const u32 k = b + ctz64(hit);
+            word |= (old & ~lowmask(k)) | (lowmask(k) & ~lowmask(b));
+            met = true;
+            break;
+          }
+          word |= lowmask(n) << b;
+          pos += coded ? sync_block<S, D>(r, a.z) : n;
+        }
+        a.marks[cur] = word;
+        cur++;
+      }
+      if (!met) {
+        for (; round && cur < (end + 63) >> 6; cur++)
+          a.marks[cur] = 0;
+        out = a.at + pos;
+      }
+    }
+    a.start_new[i] = t;
+    a.exit_new[i] = out;
+  }
+  const u64 m = __ballot(open);
+  if (m && threadIdx.x == ctz64(m))
+    atomicMin(&a.state->open[round - 1], i);
+}
+
+// marks per tile of 64 words, a wave each
+template <int UNUSED = 0>
+__global__ void __launch_bounds__(256)
+k_marks_count(const u64* __restrict__ marks, u32 tiles, u64* __restrict__ counts)
+{
+  const u32 t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
+  if (t > tiles)
+    return;
+  u32 c = t < tiles ? (u32)__builtin_popcountll(marks[(u64)t * 64 + lane]) : 0u;
+  for (u32 d = 32; d; d >>= 1)
+    c += __shfl_xor(c, d, 64);
+  if (lane == 0)
+    counts[t] = c; // counts[tiles] = 0, for the scan
+}
+
+// the chunk's block offsets, block k0 + j from its j-th mark; the position
+// after the last mark is the last segment's exit
+template <int UNUSED = 0>
+__global__ void __launch_bounds__(256)
+k_marks_offsets(const u64* __restrict__ marks, u32 tiles, const u64* __restrict__ first, u64 at, u64 k0,
+                u64 nblocks, u64* __restrict__ boffs, const u64* __restrict__ last_exit, SyncState* state)
+{
+  const u32 t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
+  if (t >= tiles)
+    return;
+  u64 v = marks[(u64)t * 64 + lane];
+  const u32 c = (u32)__builtin_popcountll(v);
+  u32 incl = c;
+#pragma unroll
+  for (u32 d = 1; d < 64; d <<= 1) {
+    const u32 u = __shfl_up(incl, d, 64);
+    if (lane >= d)
+      incl += u;
+  }
+  u64 k = k0 + first[t] + incl - c;
+  for (; v && k <= nblocks; v &= v - 1, k++)
+    boffs[k] = at + ((u64)t * 64 + lane) * 64 + ctz64(v);
+  if (t == 0 && lane == 0) {
+    const u64 total = first[tiles], e = *last_exit;
+    state->total = total;
+    state->exit = e;
+    if (k0 + total <= nblocks)
+      boffs[k0 + total] = e;
+  }
+}
+
+// Block offsets (nblocks + 1) of a lossy variable-length float stream of one
+// to three dimensions, chunk by chunk of the stream (256 MiB of it and its
+// marks, less when that much is not to be had).  Returns CHAIN_FALLBACK when
+// the stream holds fewer than nblocks blocks or a chunk does not settle.
+// Waits for `st`.
+template <typename S, int D>
+int sync_parse(const Desc& d, const Params& z, const u64* in, u64 nwords, u64 offset, u64* boffs, hipStream_t st)
+{
+  const u64 span = nwords * 64 > offset ? nwords * 64 - offset : 0;
+  if (!span || z.maxbits == 0 || d.nblocks == 0)
+    return CHAIN_FALLBACK;
+  // the longest block, and the average one (at most: bits past the stream's
+  // end count too)
+  const u64 longest = block_bits_bound<S, D, false>(z);
+  const u64 mean = std::min(longest, span / d.nblocks + 1);
+  // 16 blocks per segment, fewer in small fields, which do not fill the chip
+  const u64 per = std::min(16u, std::max(8u, d.nblocks >> 12));
+  const u64 L = std::max<u64>(512, (per * mean + 63) & ~63ull);
+  u64 chunk = std::min<u64>(span, 1ull << 31);
+  void* p = nullptr;
+  u64 segs, tiles;
+  for (;; chunk /= 2) {
+    if (chunk < span)
+      chunk = std::max<u64>(1, chunk / (64 * L)) * (64 * L); // whole segments and tiles
+    segs = (chunk + L - 1) / L;
+    tiles = (chunk + 4095) / 4096;
+    const int rc = g_stage.get(sizeof(SyncState) + (4 * segs + 64 * tiles + 2 * (tiles + 1)) * sizeof(u64), &p);
+    if (rc == ZFP_HIP_OK)
+      break;
+    if (chunk <= 1024 * L)
+      return rc == ZFP_HIP_ENOMEM ? CHAIN_FALLBACK : rc;
+  }
+  SyncArgs a;
+  a.z = z;
+  a.in = in;
+  a.nwords = nwords;
+  a.offset = offset;
+  a.span = span;
+  a.L = L;
+  a.window = (u32)std::min(longest + 64, L);
+  a.need = (u32)std::min<u64>(mean + 64, 64 * (SYNC_WORDS - 1));
+  a.hops = mean > 256 ? 3 : 2; // more bits to try per segment, more chances
+  a.state = (SyncState*)p;
+  u64* arr = (u64*)(a.state + 1);
+  u64* start[2] = {arr, arr + segs};
+  u64* ex[2] = {arr + 2 * segs, arr + 3 * segs};
+  a.marks = arr + 4 * segs;
+  u64* counts = a.marks + 64 * tiles;
+  u64* first = counts + tiles + 1;
+  u64 done = 0; // blocks found
+  a.entry = 0;
+  for (a.at = 0; a.at < span; a.at += a.bits) {
+    a.bits = std::min(chunk, span - a.at);
+    a.P = (u32)((a.bits + L - 1) / L);
+    const u32 T = (u32)((a.bits + 4095) / 4096);
+    a.samples = std::min(a.P, SYNC_SAMPLES);
+    a.step = a.P / a.samples;
+    HIPCHK(hipMemsetAsync(a.state, 0, offsetof(SyncState, open), st));
+    int cur = 0; // start[cur] and ex[cur] hold the latest
+    a.start_new = start[1];
+    if (a.P > 1) {
+      hipLaunchKernelGGL((k_sync_sample<S, D>), dim3(a.samples), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((k_sync_range<S>), dim3(1), dim3(64), 0, st, a);
+    }
+    // a wave per segment as long as that leaves the chip room
+    if (a.P <= 4096)
+      hipLaunchKernelGGL((k_sync_guess<S, D, 64>), dim3(a.P), dim3(64), 0, st, a);
+    else
+      hipLaunchKernelGGL((k_sync_guess<S, D, 8>), dim3(grid_for(a.P, 8)), dim3(64), 0, st, a);
+    if (a.P > 1)
+      hipLaunchKernelGGL((k_sync_retry<S, D>), dim3(std::min(a.P, 2048u)), dim3(64), 0, st, a);
+    auto walk = [&](u32 round) {
+      a.start_prev = start[cur ^ 1];
+      a.exit_prev = ex[cur ^ 1];
+      a.start_new = start[cur];
+      a.exit_new = ex[cur];
+      hipLaunchKernelGGL((k_sync_walk<S, D>), dim3(grid_for(a.P, 64)), dim3(64), 0, st, a, round);
+    };
+    walk(0);
+    struct { u32 missed, open[SYNC_ROUNDS]; u64 total, exit; } h; // the state from `missed` on
+    for (u32 look = 0;; look++) {
+      if (look == SYNC_LOOKS)
+        return CHAIN_FALLBACK;
+      if (a.P > 1) {
+        HIPCHK(hipMemsetAsync(a.state->open, 0xff, sizeof(a.state->open), st));
+        for (u32 round = 1; round <= SYNC_ROUNDS; round++) {
+          cur ^= 1;
+          walk(round);
+        }
+      }
+      hipLaunchKernelGGL(k_marks_count<0>, dim3(grid_for((u64)T + 1, 4)), dim3(256), 0, st, (const u64*)a.marks, T,
+                         counts);
+      HIPCHK(hipGetLastError());
+      int rc = exclusive_scan(counts, first, (u64)T + 1, st);
+      if (rc)
+        return rc;
+      hipLaunchKernelGGL(k_marks_offsets<0>, dim3(grid_for(T, 4)), dim3(256), 0, st, (const u64*)a.marks, T,
+                         (const u64*)first, a.at, done, (u64)d.nblocks, boffs, (const u64*)(ex[cur] + a.P - 1),
+                         a.state);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(&h, &a.state->missed, sizeof(h), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+      const u32 m = a.P > 1 ? h.open[SYNC_ROUNDS - 1] : ~0u;
+      if (m == ~0u)
+        break;
+      if (h.missed > a.P / 2)
+        return CHAIN_FALLBACK;
+      // segments 0 .. m are settled: enough when the field ends in them
+      // (what follows a stream in its buffer need not settle)
+      u64 before = 0;
+      HIPCHK(hipMemcpyAsync(&before, first + std::min((u64)(m + 1) * L, a.bits) / 4096, sizeof(u64), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+      if (done + before > d.nblocks)
+        return ZFP_HIP_OK;
+    }
+    done += h.total;
+    if (done >= d.nblocks)
+      return ZFP_HIP_OK;
+    a.entry = h.exit;
+  }
+  return CHAIN_FALLBACK;
+}
+
+} // namespace zfphip
