@@ -1114,47 +1114,50 @@ struct SlotPlaneEncoder {
     // the n significant coefficients' bits verbatim; r: the others' bits
     const u64 sig = lowmask(n);
     const u64 r = (x & ~sig) >> (n & 63u);
-    const bool all = n >= (u32)N;
-    const bool nz = r != 0;
-    const u32 m = (u32)__builtin_popcountll(r);
-    const u32 pm = nz ? 63u - (u32)__builtin_clzll(r) : 0u;
-    const bool implied = nz && n + pm + 1 >= (u32)N;
+    u32 lo = (u32)r, hi = (u32)(r >> 32);
+    const u32 m0 = (u32)__builtin_popcount(lo), m = m0 + (u32)__builtin_popcount(hi);
+    const u32 top = r ? 64u - (u32)__builtin_clzll(r) : 0u; // up to the highest one-bit
     // group-test code: bit 0 the first test; the j-th one-bit of r (at p)
     // at p + j, then the next test (a 1) at p + j + 1; the last one-bit is
     // followed by a 0 test, or is itself implied (not written) when it is
     // the last coefficient
-    const u32 keep = nz ? (implied ? pm + m : pm + m + 1) : 0u;
-    const u32 glen = all ? 0u : !nz ? 1u : (implied ? pm + m : pm + m + 2);
-    u64 c0 = nz ? 1ull : 0ull, c1 = 0;
-    if (wave_any(nz && pm + m >= 63)) {
-      // some lane's code reaches past bit 63
-      u64 rr = r;
-      for (u32 j = 1; wave_any(rr != 0); j++) {
-        if (rr) {
-          const u32 s = ctz64(rr) + j;   // < 128
-          xor128(c0, c1, 3ull, s);
-          rr &= rr - 1;
+    const bool rest = n + top < (u32)N;
+    const u32 keep = r ? (rest ? top + m : top + m - 1) : 0u;
+    const u32 glen = keep + (rest ? 1u : 0u);
+    // the one-bits of each half of r in turn: those of the upper half lie
+    // 32 + m0 bits further than they would by themselves
+    u64 c0 = r ? 1ull : 0ull, c1 = 0;
+    for (u32 j = 1; wave_any(lo != 0); j++) {
+      if (lo) {
+        c0 |= 3ull << ((u32)__builtin_ctz(lo) + j); // <= 63
+        lo &= lo - 1;
+      }
+    }
+    if (wave_any(hi != 0)) {
+      u64 h = 0;
+      for (u32 j = 1; wave_any(hi != 0); j++) {
+        if (hi) {
+          h |= 3ull << ((u32)__builtin_ctz(hi) + j);
+          hi &= hi - 1;
         }
       }
-      c1 &= lowmask(keep > 64 ? keep - 64 : 0u);
-      c0 &= lowmask(keep);
+      c0 |= (h << 32) << m0;
+      // 32 one-bits in the lower half: the test after the last is bit 64
+      c1 = (h >> (32 - m0)) | (m0 >> 5);
     }
-    else {
-      u64 rr = r;
-      for (u32 j = 1; wave_any(rr != 0); j++) {
-        if (rr) {
-          c0 |= 3ull << (ctz64(rr) + j);   // < 64
-          rr &= rr - 1;
-        }
+    c0 &= lowmask(keep);
+    if (wave_any(n + glen > 64)) {
+      w.put(x & sig, n);
+      w.put(c0, umin(glen, 64u));
+      if (wave_any(glen > 64)) {
+        c1 &= lowmask(keep > 64 ? keep - 64 : 0u);
+        w.put(c1, glen > 64 ? glen - 64 : 0u);
       }
-      c0 &= lowmask(keep);
     }
-    w.put(x & sig, all ? (u32)N : n);
-    w.put(c0, umin(glen, 64u));
-    if (wave_any(glen > 64))
-      w.put(c1, glen > 64 ? glen - 64 : 0u);
-    pos += (all ? (u32)N : n) + glen;
-    n += nz ? pm + 1 : 0u;
+    else
+      w.put((x & sig) | (c0 << (n & 63u)), n + glen);
+    pos += n + glen;
+    n += top;
   }
 };
 
