@@ -1,7 +1,7 @@
 // codec_sync.h -- block starts of a variable-length float stream that arrives
 // without an index, from guessed starts that are then proven.
 //
-// The stream's bits are cut into segments of about SYNC_BLOCKS blocks, one
+// The stream's bits are cut into segments of 8 to 16 blocks on average, one
 // lane each.  A segment's lane can only follow block lengths once it knows
 // where some block starts, and a chain of lengths from an arbitrary bit meets
 // the true one only after about as many blocks as a block has bits.  A block
