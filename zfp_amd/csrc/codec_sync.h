@@ -607,8 +607,6 @@ int sync_parse(const Desc& d, const Params& z, const u64* in, u64 nwords, u64 of
       const u32 m = a.P > 1 ? h.open[SYNC_ROUNDS - 1] : ~0u;
       if (m == ~0u)
         break;
-      if (h.missed > a.P / 2)
-        return CHAIN_FALLBACK;
       // segments 0 .. m are settled: enough when the field ends in them
       // (what follows a stream in its buffer need not settle)
       u64 before = 0;
@@ -616,6 +614,8 @@ int sync_parse(const Desc& d, const Params& z, const u64* in, u64 nwords, u64 of
       HIPCHK(hipStreamSynchronize(st));
       if (done + before > d.nblocks)
         return ZFP_HIP_OK;
+      if (h.missed > a.P / 2)
+        return CHAIN_FALLBACK;
     }
     done += h.total;
     if (done >= d.nblocks)
